@@ -36,23 +36,31 @@ constexpr int SCORE_PASSES = 4;  // pages per scoring thread
 __host__ __device__ inline int64_t score_stride(int max_done) { return (max_done + 3) & ~3; }
 constexpr int TOPK_LDS_KEYS = 15360;  // rows of at most this many committed pages select from keys held in LDS (60 KiB)
 
-// One wave per (row b, Quest page first + i, KV head).
-template <int FMT>
+// One wave per (row b, kBoundsPages Quest pages, KV head): enough pages that a wave's loads of the next page overlap
+// the reduction of the current one.
+constexpr int kBoundsPages = 4;
+
+template <int FMT, int D>
 __global__ __launch_bounds__(64) void quest_bounds_kernel(BoundsParams p) {
-    const int pages = p.last - p.first;
-    quest_bounds_of_page<FMT>(p, blockIdx.x / pages, p.first + blockIdx.x % pages, blockIdx.y, threadIdx.x);
+    const int chunks = (p.last - p.first + kBoundsPages - 1) / kBoundsPages;
+    const int q0 = p.first + static_cast<int>(blockIdx.x % chunks) * kBoundsPages;
+    quest_bounds_range<FMT, D>(p, blockIdx.x / chunks, blockIdx.y, q0, min(q0 + kBoundsPages, p.last), threadIdx.x);
 }
 
 // The bounds of the pages each (row, KV head) committed since its last refresh, with every range on the device (a
-// launch of fixed shape, so a decode step that keeps its Quest metadata can be captured in a graph): workgroup
-// (b * Hkv + h, y) takes pages valid + y, valid + y + Y, ... below the row's committed pages.
-template <int FMT>
-__global__ __launch_bounds__(64) void quest_refresh_kernel(BoundsParams p) {
+// launch of fixed shape, so a decode step that keeps its Quest metadata can be captured in a graph): the waves of row
+// b * Hkv + h take equal contiguous parts of its pages from valid up to the committed ones.
+template <int FMT, int D>
+__global__ __launch_bounds__(256) void quest_refresh_kernel(BoundsParams p) {
     const int row = blockIdx.x;
     const int b = row / p.kv_heads, kvh = row % p.kv_heads;
     const int last = min(max(p.committed[b], 0) / (16 * p.span), p.page_cap);
-    for (int qp = p.valid[row] + static_cast<int>(blockIdx.y); qp < last; qp += gridDim.y)
-        quest_bounds_of_page<FMT>(p, b, qp, kvh, threadIdx.x);
+    const int from = p.valid[row];
+    const int waves = static_cast<int>(gridDim.y) * 4;
+    const int wave = static_cast<int>(blockIdx.y) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int each = (last - from + waves - 1) / waves;
+    const int q0 = from + wave * each;
+    quest_bounds_range<FMT, D>(p, b, kvh, q0, min(q0 + each, last), threadIdx.x & 63);
 }
 
 // After quest_refresh_kernel (the next launch on the stream): the refreshed pages are final, and done[b] is the
@@ -526,13 +534,11 @@ int quest_score_chunk(int head_dim) {
 
 int quest_bounds(const BoundsParams& p, hipStream_t stream) {
     if (p.last <= p.first) return 0;
-    dim3 grid(static_cast<unsigned>(p.batch) * (p.last - p.first), p.kv_heads);
-    switch (p.kv_format) {
-        case BF16: hipLaunchKernelGGL(quest_bounds_kernel<BF16>, grid, dim3(64), 0, stream, p); break;
-        case FP8_E4M3: hipLaunchKernelGGL(quest_bounds_kernel<FP8_E4M3>, grid, dim3(64), 0, stream, p); break;
-        case FP8_E5M2: hipLaunchKernelGGL(quest_bounds_kernel<FP8_E5M2>, grid, dim3(64), 0, stream, p); break;
-        default: return fail("quest page bounds: KV format must be bf16, fp8 e4m3 or fp8 e5m2");
-    }
+    dim3 grid(static_cast<unsigned>(p.batch) * ((p.last - p.first + kBoundsPages - 1) / kBoundsPages), p.kv_heads);
+    if (!quest_bounds_dispatch(p.kv_format, p.head_dim, [&](auto fmt, auto dim) {
+            hipLaunchKernelGGL((quest_bounds_kernel<fmt.value, dim.value>), grid, dim3(64), 0, stream, p);
+        }))
+        return fail("quest page bounds: KV format must be bf16, fp8 e4m3 or fp8 e5m2");
     return check_launch("quest_bounds_kernel");
 }
 
@@ -554,17 +560,23 @@ int quest_dense_bounds(const DenseBoundsParams& p, hipStream_t stream) {
     return check_launch("quest_dense_bounds_kernel");
 }
 
+// Waves per (row, KV head) of the refresh: enough to fill the chip when a prompt's pages are due (about 4096 waves),
+// with at least four pages of the bounds' capacity each; never under eight, the shape of a decode step, whose rows
+// complete at most one page.
+static int refresh_waves(int rows, int page_cap) {
+    const int fill = 4096 / rows, due = page_cap / 4;
+    const int waves = fill < due ? fill : due;
+    return waves < 8 ? 8 : (waves + 3) / 4 * 4;
+}
+
 int quest_refresh(const BoundsParams& p, hipStream_t stream) {
     const int rows = p.batch * p.kv_heads;
     if (rows == 0) return 0;
-    constexpr int CHUNKS = 8;  // waves per (row, KV head): a decode step completes at most one page per row
-    dim3 grid(rows, CHUNKS);
-    switch (p.kv_format) {
-        case BF16: hipLaunchKernelGGL(quest_refresh_kernel<BF16>, grid, dim3(64), 0, stream, p); break;
-        case FP8_E4M3: hipLaunchKernelGGL(quest_refresh_kernel<FP8_E4M3>, grid, dim3(64), 0, stream, p); break;
-        case FP8_E5M2: hipLaunchKernelGGL(quest_refresh_kernel<FP8_E5M2>, grid, dim3(64), 0, stream, p); break;
-        default: return fail("quest refresh: KV format must be bf16, fp8 e4m3 or fp8 e5m2");
-    }
+    dim3 grid(rows, refresh_waves(rows, p.page_cap) / 4);
+    if (!quest_bounds_dispatch(p.kv_format, p.head_dim, [&](auto fmt, auto dim) {
+            hipLaunchKernelGGL((quest_refresh_kernel<fmt.value, dim.value>), grid, dim3(256), 0, stream, p);
+        }))
+        return fail("quest refresh: KV format must be bf16, fp8 e4m3 or fp8 e5m2");
     if (int rc = check_launch("quest_refresh_kernel")) return rc;
     hipLaunchKernelGGL(quest_mark_kernel, dim3((rows + 255) / 256), dim3(256), 0, stream, p);
     return check_launch("quest_mark_kernel");

@@ -36,6 +36,14 @@ ECO_HD constexpr float fp8_max() {
 // of its operands, which the compiler otherwise inserts wherever it cannot prove an operand is not a signalling NaN.
 __device__ inline float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
+__device__ inline float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+
+// x of the lane a DPP control names (its lanes all in range).
+template <int CTRL>
+__device__ inline uint32_t dpp(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xF, 0xF, true));
+}
+
 __device__ inline float group_max(float x) {  // max over the four lanes l, l^16, l^32, l^48 (NaN if any is NaN)
     x = max_nan(x, __shfl_xor(x, 16));
     return max_nan(x, __shfl_xor(x, 32));

@@ -1,13 +1,5 @@
-// KIVI (Liu et al., ICML 2024) on gfx950: the quantization schedule, the full-precision residual ring,
-// quantize-and-append into 32-token pages, and decode attention that feeds the codes to the matrix cores.
-//
-// Quantization follows the reference's quantize (techniques/kv_quant/kivi.py:121-140): fp32 min and max along the
-// group; scale = fp16r((high - low) / levels) and low = fp16r(low), fp16r rounding to nearest even where fp16 holds
-// the value; codes = round_half_even((x - low) / safe) clamped to [0, levels], safe = scale or 1 where the scale is 0.
-// Both divisions are IEEE divisions (__fdiv_rn), the CPU semantics of torch's tensor / int and tensor / tensor (GPU
-// torch multiplies by a reciprocal instead; the parity oracle is the CPU definition). Keys are quantized per channel
-// over a 32-token group (one page), values per token over 32-channel groups. The schedule is the reference's
-// (kivi.py:230-243): with c committed tokens, keys below (c / R) * R and values below max(0, c - R) are quantized.
+// KIVI (Liu et al., ICML 2024) on gfx950: decode attention that feeds the codes to the matrix cores (the pages and the
+// residual ring are written by kivi_quantize.hip).
 //
 // Page block (one per (page, KV head), offsets in KiviLayout): key codes token-major, each token's channels packed
 // in 32-bit words; value codes as words (u * 16 + n) * (D / 16) + nd, channel 16 nd + n, tokens u * 32 / bits ..;
@@ -40,159 +32,6 @@ namespace eco {
 namespace {
 
 constexpr int KPAGE = KiviParams::kPage;  // 32 tokens
-
-__device__ inline float load_elem(const void* base, int64_t offset, int format) {
-    if (format == BF16) return bf16_to_f32(static_cast<const uint16_t*>(base)[offset]);
-    if (format == FP16) return static_cast<float>(static_cast<const _Float16*>(base)[offset]);
-    return static_cast<const float*>(base)[offset];
-}
-
-__device__ inline uint16_t f16_bits(float x) {
-    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
-}
-
-// ---- schedule --------------------------------------------------------------------------------------------------
-
-// ranges [4][B]: keys [from, to), values [from, to) to quantize now; the counts advance to their new values.
-__global__ void kivi_schedule_kernel(const int32_t* committed, int residual, int32_t* kq, int32_t* vq,
-                                     int32_t* ranges, int batch) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= batch) return;
-    const int c = max(committed[b], 0);
-    const int k_to = max(kq[b], (c / residual) * residual);
-    const int v_to = max(vq[b], c - residual);
-    ranges[b] = kq[b];
-    ranges[batch + b] = k_to;
-    ranges[2 * batch + b] = vq[b];
-    ranges[3 * batch + b] = v_to;
-    kq[b] = k_to;
-    vq[b] = v_to;
-}
-
-// ---- residual ring ------------------------------------------------------------------------------------------
-
-// One workgroup per new token: keys to slot t % W of [B, Hkv, W, D], values to [B, Hkv, D, W], rounded to bf16.
-__global__ __launch_bounds__(256) void kivi_ring_kernel(KiviRingParams p) {
-    const int t = blockIdx.x;
-    const int pos = p.positions[t];
-    const int b = p.rows[t];
-    if (pos < 0 || b < 0 || b >= p.batch) return;
-    const int slot = pos % p.ring;
-    for (int i = threadIdx.x; i < p.kv_heads * p.head_dim; i += blockDim.x) {
-        const int h = i / p.head_dim, d = i % p.head_dim;
-        const float k = load_elem(p.k_new, t * p.sk_t + h * p.sk_h + d, p.in_format);
-        const float v = load_elem(p.v_new, t * p.sv_t + h * p.sv_h + d, p.in_format);
-        const int64_t row = static_cast<int64_t>(b) * p.kv_heads + h;
-        p.k_ring[(row * p.ring + slot) * p.head_dim + d] = f32_to_bf16(k);
-        p.v_ring[(row * p.head_dim + d) * p.ring + slot] = f32_to_bf16(v);
-    }
-}
-
-// ---- quantize-and-append ----------------------------------------------------------------------------------------
-
-__device__ inline float src_elem(const KiviQuantParams& p, int b, int h, int t, int d) {
-    const int slot = p.src_ring > 0 ? t % p.src_ring : t - p.src_start;
-    return load_elem(p.src, b * p.ss_b + h * p.ss_h + static_cast<int64_t>(slot) * p.ss_t + d * p.ss_d,
-                     p.src_format);
-}
-
-__device__ inline uint8_t* page_block(const KiviQuantParams& p, int b, int h, int page) {
-    if (page >= p.bt_cols) return nullptr;
-    const int phys = p.block_table[b * p.bt_stride + page];
-    if (phys < 0 || phys >= p.num_pages) return nullptr;
-    return p.blocks + static_cast<int64_t>(phys) * p.blk_page + h * p.blk_head;
-}
-
-// Keys: one workgroup per (row, KV head) and 32-token group in [from, to) (multiples of 32).
-__global__ __launch_bounds__(256) void kivi_quant_keys_kernel(KiviQuantParams p) {
-    __shared__ float s_low[256], s_safe[256];
-    const int row = blockIdx.x;
-    const int b = row / p.kv_heads, h = row % p.kv_heads;
-    const int page = p.from[b] / KPAGE + static_cast<int>(blockIdx.y);
-    const int t0 = page * KPAGE;
-    if (t0 + KPAGE > p.to[b]) return;
-    uint8_t* blk = page_block(p, b, h, page);
-    if (!blk) return;
-    const KiviLayout L{p.head_dim, p.bits};
-    const int levels = (1 << p.bits) - 1;
-    for (int d = threadIdx.x; d < p.head_dim; d += blockDim.x) {
-        float lo = INFINITY, hi = -INFINITY;
-        for (int t = 0; t < KPAGE; ++t) {
-            const float x = src_elem(p, b, h, t0 + t, d);
-            lo = fminf(lo, x);
-            hi = fmaxf(hi, x);
-        }
-        const Quant q = make_quant(lo, hi, levels, p.overflow);
-        s_low[d] = q.low;
-        s_safe[d] = q.safe;
-        reinterpret_cast<uint16_t*>(blk + L.k_scale())[d] = f16_bits(q.scale);
-        reinterpret_cast<uint16_t*>(blk + L.k_zero())[d] = f16_bits(q.low);
-    }
-    __syncthreads();
-    const int per_word = 32 / p.bits;
-    const int words = p.head_dim / per_word;  // per token
-    for (int item = threadIdx.x; item < KPAGE * words; item += blockDim.x) {
-        const int t = item / words, w = item % words;
-        uint32_t word = 0;
-        for (int e = 0; e < per_word; ++e) {
-            const int d = w * per_word + e;
-            const Quant q{0.0f, s_low[d], s_safe[d]};
-            word |= code_of(src_elem(p, b, h, t0 + t, d), q, levels) << (8 * (e & 3) + (e >> 2) * p.bits);
-        }
-        reinterpret_cast<uint32_t*>(blk + L.k_codes() + t * (p.head_dim * p.bits / 8))[w] = word;
-    }
-}
-
-// Values: one workgroup per (row, KV head) and page overlapping [from, to); the page's other tokens keep their codes.
-__global__ __launch_bounds__(256) void kivi_quant_values_kernel(KiviQuantParams p) {
-    __shared__ float s_low[KPAGE][8], s_safe[KPAGE][8];
-    const int row = blockIdx.x;
-    const int b = row / p.kv_heads, h = row % p.kv_heads;
-    const int page = p.from[b] / KPAGE + static_cast<int>(blockIdx.y);
-    const int t0 = page * KPAGE;
-    const int lo_t = max(p.from[b], t0), hi_t = min(p.to[b], t0 + KPAGE);
-    if (lo_t >= hi_t) return;
-    uint8_t* blk = page_block(p, b, h, page);
-    if (!blk) return;
-    const KiviLayout L{p.head_dim, p.bits};
-    const int levels = (1 << p.bits) - 1;
-    const int groups = p.head_dim / 32;
-    for (int item = threadIdx.x; item < (hi_t - lo_t) * groups; item += blockDim.x) {
-        const int t = lo_t + item / groups, grp = item % groups;
-        float lo = INFINITY, hi = -INFINITY;
-        for (int d = 32 * grp; d < 32 * grp + 32; ++d) {
-            const float x = src_elem(p, b, h, t, d);
-            lo = fminf(lo, x);
-            hi = fmaxf(hi, x);
-        }
-        const Quant q = make_quant(lo, hi, levels, p.overflow);
-        s_low[t - t0][grp] = q.low;
-        s_safe[t - t0][grp] = q.safe;
-        reinterpret_cast<uint16_t*>(blk + L.v_scale())[grp * KPAGE + (t - t0)] = f16_bits(q.scale);
-        reinterpret_cast<uint16_t*>(blk + L.v_zero())[grp * KPAGE + (t - t0)] = f16_bits(q.low);
-    }
-    __syncthreads();
-    const int per_word = 32 / p.bits;  // tokens per word
-    const int nd_count = p.head_dim / 16;
-    uint32_t* words = reinterpret_cast<uint32_t*>(blk + L.v_codes());
-    for (int item = threadIdx.x; item < p.bits * 16 * nd_count; item += blockDim.x) {
-        const int u = item / (16 * nd_count);
-        const int n = (item / nd_count) % 16;
-        const int nd = item % nd_count;
-        const int d = 16 * nd + n;
-        const int w0 = t0 + u * per_word;  // first token of the word
-        if (w0 + per_word <= lo_t || w0 >= hi_t) continue;
-        uint32_t word = words[item];
-        for (int e = 0; e < per_word; ++e) {
-            const int t = w0 + e;
-            if (t < lo_t || t >= hi_t) continue;
-            const int shift = 8 * (e & 3) + (e >> 2) * p.bits;
-            const Quant q{0.0f, s_low[t - t0][d / 32], s_safe[t - t0][d / 32]};
-            word = (word & ~(static_cast<uint32_t>(levels) << shift)) | (code_of(src_elem(p, b, h, t, d), q, levels) << shift);
-        }
-        words[item] = word;
-    }
-}
 
 // ---- attention ----------------------------------------------------------------------------------------------
 
@@ -837,29 +676,6 @@ struct KiviOccupancy {
 };
 
 }  // namespace
-
-int kivi_schedule(const int32_t* committed, int residual, int32_t* keys_quantized, int32_t* values_quantized,
-                  int32_t* ranges, int batch, hipStream_t stream) {
-    hipLaunchKernelGGL(kivi_schedule_kernel, dim3((batch + 255) / 256), dim3(256), 0, stream, committed, residual,
-                       keys_quantized, values_quantized, ranges, batch);
-    return check_launch("kivi_schedule_kernel");
-}
-
-int kivi_ring_write(const KiviRingParams& p, hipStream_t stream) {
-    if (p.tokens == 0) return 0;
-    hipLaunchKernelGGL(kivi_ring_kernel, dim3(p.tokens), dim3(256), 0, stream, p);
-    return check_launch("kivi_ring_kernel");
-}
-
-int kivi_quantize(const KiviQuantParams& p, int kind, int max_tokens, hipStream_t stream) {
-    const int pages = (max_tokens + KPAGE - 1) / KPAGE + 1;  // a range need not start at a page boundary
-    dim3 grid(p.batch * p.kv_heads, pages);
-    if (kind == 0)
-        hipLaunchKernelGGL(kivi_quant_keys_kernel, grid, dim3(256), 0, stream, p);
-    else
-        hipLaunchKernelGGL(kivi_quant_values_kernel, grid, dim3(256), 0, stream, p);
-    return check_launch(kind == 0 ? "kivi_quant_keys_kernel" : "kivi_quant_values_kernel");
-}
 
 int kivi_resident_groups(int head_dim, int bits, int rows, int* per_cu, int* waves) {
     return kivi_dispatch(head_dim, bits, rows, KiviOccupancy{per_cu, waves});

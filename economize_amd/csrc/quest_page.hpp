@@ -94,11 +94,6 @@ __device__ inline i16x2 ordered_bf16(i16x2 x) {
     return x ^ (sign & static_cast<short>(0x7FFF));
 }
 
-template <int CTRL>
-__device__ inline uint32_t dpp(uint32_t x) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xF, 0xF, true));
-}
-
 // Halves v[0 .. 2 N): the lane keeps the half its `upper` names, sends the other to its partner (a lane permutation
 // that is its own inverse and pairs lanes of different `upper`) and takes the minimum with what the partner sent.
 template <int CTRL, int N>

@@ -75,6 +75,27 @@ __device__ inline float soft_cap_log2(float x, float cap, float inv_cap) {
     return cap * kLog2e * (t < 0.0f ? -th : th);
 }
 
+// Two (eight) bf16 or fp16 values of a word (four words) as floats, exactly.
+template <int FMT>
+__device__ __forceinline__ void unpack_pair(uint32_t w, float& a, float& b) {
+    if constexpr (FMT == BF16) {
+        a = bits_f32(w << 16);
+        b = bits_f32(w & 0xFFFF0000u);
+    } else {
+        const f16x2 h = __builtin_bit_cast(f16x2, w);
+        a = static_cast<float>(h[0]);
+        b = static_cast<float>(h[1]);
+    }
+}
+
+template <int FMT>
+__device__ __forceinline__ void unpack8(const uint4& w, float (&x)[8]) {
+    unpack_pair<FMT>(w.x, x[0], x[1]);
+    unpack_pair<FMT>(w.y, x[2], x[3]);
+    unpack_pair<FMT>(w.z, x[4], x[5]);
+    unpack_pair<FMT>(w.w, x[6], x[7]);
+}
+
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // A 16-byte load of cache data read once per call (K/V tiles, codes): nontemporal, so the line is streamed rather than

@@ -187,26 +187,6 @@ __global__ __launch_bounds__(256) void kivi_quant_values_kernel(KiviQuantParams 
 // gives the same codes (page_code). 8 rows x 4096 tokens x 8 KV heads, D = 128, 4 bits, bf16 (84 MB each): keys 119 and
 // values 120 us by workgroups, 31 us together by waves (5.4 TB/s).
 
-template <int FMT>
-__device__ __forceinline__ void unpack_pair(uint32_t w, float& a, float& b) {
-    if constexpr (FMT == BF16) {
-        a = bits_f32(w << 16);
-        b = bits_f32(w & 0xFFFF0000u);
-    } else {
-        const f16x2 h = __builtin_bit_cast(f16x2, w);
-        a = static_cast<float>(h[0]);
-        b = static_cast<float>(h[1]);
-    }
-}
-
-template <int FMT>
-__device__ __forceinline__ void unpack8(const uint4& w, float (&x)[8]) {
-    unpack_pair<FMT>(w.x, x[0], x[1]);
-    unpack_pair<FMT>(w.y, x[2], x[3]);
-    unpack_pair<FMT>(w.z, x[4], x[5]);
-    unpack_pair<FMT>(w.w, x[6], x[7]);
-}
-
 // A group's quantization with what its codes need.
 struct PageQuant {
     float scale, low, safe, rcp;

@@ -34,6 +34,60 @@ __device__ inline uint8_t encode(float x, float scale, bool scaled) {
     return f32_to_fp8<FMT>(fminf(fmaxf(w, -fp8_max<FMT>()), fp8_max<FMT>()));
 }
 
+// ---- encoding four values at a time -------------------------------------------------------------------------------
+//
+// What encode() computes, for bf16 and fp16 inputs: x / s as corrected_quotient and the hardware's round-to-nearest-even
+// conversion of two values per instruction, about 6 operations per value instead of 30. The quotient is IEEE division's for every 8- or 11-bit
+// significand of x and every fp32 significand of s (checked exhaustively) while nothing under- or overflows, which
+// kScaleMin <= s <= kScaleMax and |x| < 2^60 ensure down to |x| = 2^-64; a smaller |x| gives a quotient below 2^-23, a zero
+// of x's sign in both formats either way. The conversion equals f32_to_fp8 on every fp32 value up to the format's maximum
+// (checked on all of them). Values outside these limits (and NaN) take encode().
+constexpr float kScaleMin = 0x1p-40f, kScaleMax = 0x1p60f;
+
+template <int FMT>
+__device__ __forceinline__ uint32_t fp8_pack4(float a, float b, float c, float d) {
+    if constexpr (FMT == FP8_E4M3)
+        return static_cast<uint32_t>(
+            __builtin_amdgcn_cvt_pk_fp8_f32(c, d, __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false), true));
+    else
+        return static_cast<uint32_t>(
+            __builtin_amdgcn_cvt_pk_bf8_f32(c, d, __builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false), true));
+}
+
+// Codes of four values. FAST: within the limits above; CLAMP: quotients may pass the format's maximum (they do not with
+// the scale of their own largest value, whose quotient is at most an ulp beyond it).
+template <int FMT, bool FAST, bool CLAMP>
+__device__ __forceinline__ uint32_t encode4(float a, float b, float c, float d, float s, float r) {
+    if constexpr (FAST) {
+        const auto one = [&](float x) __attribute__((always_inline)) {
+            const float q = corrected_quotient(x, s, r);
+            return CLAMP ? __builtin_amdgcn_fmed3f(q, -fp8_max<FMT>(), fp8_max<FMT>()) : q;
+        };
+        return fp8_pack4<FMT>(one(a), one(b), one(c), one(d));
+    }
+    return encode<FMT>(a, s, true) | encode<FMT>(b, s, true) << 8 | encode<FMT>(c, s, true) << 16 |
+           static_cast<uint32_t>(encode<FMT>(d, s, true)) << 24;
+}
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// The larger of two pairs of 16-bit magnitudes.
+__device__ __forceinline__ uint32_t max_pair(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// The largest magnitude's bits in the four words' eight values, in the low half.
+__device__ __forceinline__ uint32_t max_magnitude8(const uint4& w) {
+    constexpr uint32_t M = 0x7FFF7FFFu;
+    const uint32_t m = max_pair(max_pair(w.x & M, w.y & M), max_pair(w.z & M, w.w & M));
+    return max_pair(m, m >> 16) & 0xFFFFu;
+}
+
+template <int IN>
+__device__ __forceinline__ bool magnitude_within(uint32_t bits) {  // below 2^60 (fp16: finite)
+    return bits < (IN == BF16 ? 0x5D80u : 0x7C00u);
+}
+
 // New token t into its slot, by one workgroup.
 template <int FMT>
 __device__ inline void append_token(const AppendParams& p, int t) {
@@ -167,6 +221,87 @@ __global__ __launch_bounds__(256) void fp8_encode_kernel(EncodeParams p) {
     }
 }
 
+// The dense encode of bf16 and fp16 rows whose 8-channel runs are 16-byte loads and 8-byte stores: L lanes per row (D / 8
+// rounded up to a power of two), kEncodeRows rows per lane with all their loads in flight. Bound by reading x and writing
+// the codes; fp8_encode_kernel, which takes everything else, is bound by its instructions: 2-byte loads, three 64-bit
+// divisions per row, the IEEE divisions and the bitwise encoder. 8 x 8 x 4096 rows of D = 128, bf16 with a
+// scale per token (101 MB): 133 us there, 19.4 us here (5.2 TB/s).
+constexpr int kEncodeRows = 4;
+
+template <int FMT, int IN, int L>
+__global__ __launch_bounds__(256) void fp8_encode_rows_kernel(EncodeParams p) {
+    constexpr int R = 256 / L;  // rows per workgroup and step
+    const int c = threadIdx.x % L;
+    const int b = blockIdx.y / p.heads, h = blockIdx.y % p.heads;
+    const int t0 = blockIdx.x * (R * kEncodeRows) + threadIdx.x / L;
+    const bool lane_used = 8 * c < p.head_dim;
+    const uint16_t* src = static_cast<const uint16_t*>(p.src) + b * p.ss_b + h * p.ss_h + 8 * c;
+    uint8_t* dst = p.dst + b * p.sd_b + h * p.sd_h + 8 * c;
+    uint4 raw[kEncodeRows];
+#pragma unroll
+    for (int i = 0; i < kEncodeRows; ++i) {
+        const int t = t0 + i * R;
+        raw[i] = lane_used && t < p.tokens ? stream_load16(src + t * p.ss_t) : make_uint4(0, 0, 0, 0);
+    }
+    const bool per_token = p.token_scale != nullptr;
+    const float head = p.head_scale ? p.head_scale[h] : 1.0f;
+#pragma unroll
+    for (int i = 0; i < kEncodeRows; ++i) {
+        const int t = t0 + i * R;
+        if (blockIdx.x * (R * kEncodeRows) + i * R >= p.tokens) break;
+        uint32_t m = max_magnitude8(raw[i]);
+        float s = head;
+        if (per_token) {
+            m = max(m, dpp<0xB1>(m));   // quad_perm 1 0 3 2
+            m = max(m, dpp<0x4E>(m));   // quad_perm 2 3 0 1
+            m = max(m, dpp<0x141>(m));  // row_half_mirror
+            if constexpr (L > 8) m = max(m, dpp<0x140>(m));  // row_mirror
+            if constexpr (L > 16) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16)));
+            if constexpr (L > 32) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32)));
+            const float amax = IN == BF16 ? bits_f32(m << 16)
+                                          : static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(m)));
+            // a NaN's magnitude is the largest: the row's scale is then NaN, as torch's amax propagates it
+            s = amax == amax ? fmaxf(__fdiv_rn(amax, fp8_max<FMT>()), 1e-12f) : __builtin_nanf("");
+            if (c == 0 && t < p.tokens) p.token_scale[b * p.st_b + h * p.st_h + t * p.st_t] = s;
+        }
+        const bool ok = magnitude_within<IN>(m) && s >= kScaleMin && s <= kScaleMax;
+        const float r = __fdiv_rn(1.0f, s);
+        float x[8];
+        unpack8<IN>(raw[i], x);
+        uint2 codes;
+        const auto encode8 = [&](auto fast, auto clamp) __attribute__((always_inline)) {
+            constexpr bool F = decltype(fast)::value, K = decltype(clamp)::value;
+            codes.x = encode4<FMT, F, K>(x[0], x[1], x[2], x[3], s, r);
+            codes.y = encode4<FMT, F, K>(x[4], x[5], x[6], x[7], s, r);
+        };
+        if (__ballot(!ok) != 0) encode8(std::false_type{}, std::true_type{});
+        else if (per_token) encode8(std::true_type{}, std::false_type{});
+        else encode8(std::true_type{}, std::true_type{});
+        if (lane_used && t < p.tokens) *reinterpret_cast<uint2*>(dst + t * p.sd_t) = codes;
+    }
+}
+
+// Whether fp8_encode_rows_kernel takes a call: its loads and stores aligned, its grid within the limits.
+bool encode_rows(const EncodeParams& p) {
+    return (p.in_format == BF16 || p.in_format == FP16) && p.head_dim % 8 == 0 &&
+           static_cast<int64_t>(p.batch) * p.heads <= 65535 && ((p.ss_b | p.ss_h | p.ss_t) & 7) == 0 &&
+           ((p.sd_b | p.sd_h | p.sd_t) & 7) == 0 && (reinterpret_cast<uintptr_t>(p.src) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(p.dst) & 7) == 0;
+}
+
+template <int FMT, int IN>
+void launch_encode_rows(const EncodeParams& p, hipStream_t stream) {
+    const auto launch = [&](auto lanes) {
+        constexpr int L = decltype(lanes)::value;
+        const dim3 grid(ceil_div(p.tokens, 256 / L * kEncodeRows), p.batch * p.heads);
+        hipLaunchKernelGGL((fp8_encode_rows_kernel<FMT, IN, L>), grid, dim3(256), 0, stream, p);
+    };
+    if (p.head_dim <= 64) launch(std::integral_constant<int, 8>{});
+    else if (p.head_dim <= 128) launch(std::integral_constant<int, 16>{});
+    else if (p.head_dim <= 256) launch(std::integral_constant<int, 32>{});
+    else launch(std::integral_constant<int, 64>{});
+}
+
 // absmax[h] = max |x[a, h, s, d]| as float bits (non-negative floats order like their bit patterns).
 __global__ __launch_bounds__(256) void head_absmax_kernel(AbsmaxParams p) {
     const int h = blockIdx.y;
@@ -221,6 +356,12 @@ int paged_append_quest(const AppendParams& p, const BoundsParams& q, int32_t* co
 int fp8_encode(const EncodeParams& p, hipStream_t stream) {
     const int64_t rows = static_cast<int64_t>(p.batch) * p.heads * p.tokens;
     if (rows == 0) return 0;
+    if (encode_rows(p) && (p.out_format == FP8_E4M3 || p.out_format == FP8_E5M2)) {
+        const bool bf16 = p.in_format == BF16, e4m3 = p.out_format == FP8_E4M3;
+        if (bf16) e4m3 ? launch_encode_rows<FP8_E4M3, BF16>(p, stream) : launch_encode_rows<FP8_E5M2, BF16>(p, stream);
+        else e4m3 ? launch_encode_rows<FP8_E4M3, FP16>(p, stream) : launch_encode_rows<FP8_E5M2, FP16>(p, stream);
+        return check_launch("fp8_encode_rows_kernel");
+    }
     const int blocks = static_cast<int>((rows + 3) / 4 < 65535 ? (rows + 3) / 4 : 65535);
     switch (p.out_format) {
         case FP8_E4M3: hipLaunchKernelGGL(fp8_encode_kernel<FP8_E4M3>, dim3(blocks), dim3(256), 0, stream, p); break;

@@ -35,9 +35,24 @@ long codes() {
     return bad;
 }
 
+// x / s for every 8-bit x and every s, and for every 11-bit x and one s in 16, with the rounded reciprocal.
+long shared_scales() {
+    long bad = 0;
+    for (uint32_t ms = 0; ms < 1u << 23; ++ms) {
+        const float s = eco::bits_f32(0x3F800000u | ms);
+        const float r = 1.0f / s;
+        const uint32_t step = ms % 16 ? 8 : 1;
+        for (uint32_t mx = 0; mx < 1u << 10; mx += step) {
+            const float x = eco::bits_f32(0x3F800000u | mx << 13);
+            bad += eco::corrected_quotient(x, s, r) != x / s;
+        }
+    }
+    return bad;
+}
+
 }  // namespace
 
 int main() {
-    std::printf("%ld\n", constant_divisors() + codes());
+    std::printf("%ld\n", constant_divisors() + codes() + shared_scales());
     return 0;
 }

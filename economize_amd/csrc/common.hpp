@@ -96,6 +96,36 @@ __device__ __forceinline__ void unpack8(const uint4& w, float (&x)[8]) {
     unpack_pair<FMT>(w.w, x[6], x[7]);
 }
 
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// The larger of two pairs of 16-bit magnitudes.
+__device__ __forceinline__ uint32_t max_pair(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// The largest magnitude's bits in the four words' eight values, in the low half.
+__device__ __forceinline__ uint32_t max_magnitude8(const uint4& w) {
+    constexpr uint32_t M = 0x7FFF7FFFu;
+    const uint32_t m = max_pair(max_pair(w.x & M, w.y & M), max_pair(w.z & M, w.w & M));
+    return max_pair(m, m >> 16) & 0xFFFFu;
+}
+
+// bf16 pairs with their NaN quieted, as f32_to_bf16 leaves them.
+__device__ __forceinline__ uint32_t quiet_pair(uint32_t w) {
+    const uint32_t lo = (w & 0x7FFFu) > 0x7F80u ? 0x40u : 0u, hi = (w >> 16 & 0x7FFFu) > 0x7F80u ? 0x400000u : 0u;
+    return w | lo | hi;
+}
+
+template <int N>
+__device__ __forceinline__ void quiet_pairs(uint32_t (&w)[N]) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) m = max_pair(m, w[j] & 0x7FFF7FFFu);
+    if (__ballot((m & 0xFFFFu) > 0x7F80u || m >> 16 > 0x7F80u) == 0) return;
+#pragma unroll
+    for (int j = 0; j < N; ++j) w[j] = quiet_pair(w[j]);
+}
+
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // A 16-byte load of cache data read once per call (K/V tiles, codes): nontemporal, so the line is streamed rather than

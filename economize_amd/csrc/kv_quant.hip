@@ -14,6 +14,7 @@
 #include "common.hpp"
 #include "kv_quant.hpp"
 #include "quest_page.hpp"
+#include "token_window.hpp"
 
 namespace eco {
 
@@ -67,20 +68,6 @@ __device__ __forceinline__ uint32_t encode4(float a, float b, float c, float d, 
     }
     return encode<FMT>(a, s, true) | encode<FMT>(b, s, true) << 8 | encode<FMT>(c, s, true) << 16 |
            static_cast<uint32_t>(encode<FMT>(d, s, true)) << 24;
-}
-
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-// The larger of two pairs of 16-bit magnitudes.
-__device__ __forceinline__ uint32_t max_pair(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
-}
-
-// The largest magnitude's bits in the four words' eight values, in the low half.
-__device__ __forceinline__ uint32_t max_magnitude8(const uint4& w) {
-    constexpr uint32_t M = 0x7FFF7FFFu;
-    const uint32_t m = max_pair(max_pair(w.x & M, w.y & M), max_pair(w.z & M, w.w & M));
-    return max_pair(m, m >> 16) & 0xFFFFu;
 }
 
 template <int IN>
@@ -141,6 +128,195 @@ __device__ inline void append_token(const AppendParams& p, int t) {
 template <int FMT>
 __global__ __launch_bounds__(256) void paged_append_kernel(AppendParams p) {
     append_token<FMT>(p, blockIdx.x);
+}
+
+// The append by windows of 16 tokens (token_window.hpp) and units of 128 channels over the KV heads, one wave each. Bound
+// by reading the states and writing the codes; the workgroup-per-token kernel is bound by its value stores, one byte of
+// every 16-byte run from each of 16 workgroups, and by its encoder. Keys: lane (n, g) encodes a 16-byte run of token n
+// (any slots), 64 lanes writing 1 KB in a row for consecutive slots. Values: a lane holds two channels of the run's 16
+// tokens and packs each channel's run in registers, no exchange between lanes; a wave writes 2 KB in a row. Tokens outside
+// runs (decode steps, the ends of prompts) are stored alone, their loads in flight together. 32768 tokens x 8 KV heads, D
+// = 128, bf16 to e4m3 (201 MB): 250 us by token, 38.7 us by windows (5.2 TB/s).
+template <int FMT, int IN>
+__global__ __launch_bounds__(256) void paged_append_window_kernel(AppendParams p) {
+    constexpr int ES = FMT == BF16 ? 2 : 1;
+    constexpr int E = 16 / ES;           // channels per 16-byte run of the key layout
+    constexpr int KR = 128 / E / 4;      // key runs per lane
+    constexpr int KL = FMT == BF16 ? 1 : 2;  // 16-byte loads per key run
+    const int lane = threadIdx.x & 63;
+    const int first = first_of_window();
+    if (first >= p.tokens) return;
+    const unsigned channels = static_cast<unsigned>(p.kv_heads) * p.head_dim;
+    TokenWindow w = token_window(first, p.tokens, lane, [&](int t) {
+        const int slot = p.slots[t];
+        return slot / PAGE < p.num_pages ? slot : -1;
+    });
+    const uint16_t* k_new = static_cast<const uint16_t*>(p.k_new);
+    const uint16_t* v_new = static_cast<const uint16_t*>(p.v_new);
+
+    const unsigned vc = blockIdx.y * 128 + 2 * lane;  // the lane's value channels: vc, vc + 1
+    const bool v_used = vc < channels;
+    const int vh = v_used ? vc / p.head_dim : 0, vd = v_used ? vc % p.head_dim : 0;
+    const uint16_t* v_src = v_new + vh * p.sv_h + vd;
+    uint8_t* v_dst = p.v_cache + vh * p.vc_head + vd * (PAGE * ES);
+    uint32_t v[PAGE];
+    const auto load_rest = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < PAGE; ++j) {
+            v[j] = 0;
+            if (w.rest >> j & 1) v[j] = *reinterpret_cast<const uint32_t*>(v_src + (first + j) * p.sv_t);
+        }
+    };
+    if (!takes_values()) {
+        w.run = -1;
+        w.rest = 0;
+    }
+    if (w.run >= 0) {
+#pragma unroll
+        for (int j = 0; j < PAGE; ++j)
+            v[j] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(v_src + (w.run + j) * p.sv_t));
+    } else {
+        load_rest();
+    }
+
+    if (takes_keys()) {
+        const int n = lane & 15, g = lane >> 4;
+        const int slot = w.slot(first + n, first);
+        const int page = slot / PAGE, pos = slot % PAGE;
+        uint4 raw[KR][KL];
+        int h[KR], d0[KR];
+        bool used[KR];
+#pragma unroll
+        for (int i = 0; i < KR; ++i) {
+            const unsigned ch = blockIdx.y * 128 + (4 * i + g) * E;
+            used[i] = ch < channels && slot >= 0;
+            h[i] = used[i] ? ch / p.head_dim : 0;
+            d0[i] = used[i] ? ch % p.head_dim : 0;
+            const uint16_t* src = k_new + (used[i] ? (first + n) * p.sk_t : 0) + h[i] * p.sk_h + d0[i];
+#pragma unroll
+            for (int u = 0; u < KL; ++u) raw[i][u] = used[i] ? stream_load16(src + 8 * u) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < KR; ++i) {
+            uint4 out = raw[i][0];
+            if constexpr (FMT == BF16) {
+                if (__ballot(max_magnitude8(out) > 0x7F80u) != 0)
+                    out = make_uint4(quiet_pair(out.x), quiet_pair(out.y), quiet_pair(out.z), quiet_pair(out.w));
+            } else {
+                const float s = p.k_scale ? p.k_scale[h[i]] : 1.0f;
+                const bool ok = magnitude_within<IN>(max(max_magnitude8(raw[i][0]), max_magnitude8(raw[i][KL - 1]))) &&
+                                s >= kScaleMin && s <= kScaleMax;
+                const float r = __fdiv_rn(1.0f, s);
+                float x[8], y[8];
+                unpack8<IN>(raw[i][0], x);
+                unpack8<IN>(raw[i][KL - 1], y);
+                const auto run = [&](auto fast) __attribute__((always_inline)) {
+                    constexpr bool F = decltype(fast)::value;
+                    out.x = encode4<FMT, F, true>(x[0], x[1], x[2], x[3], s, r);
+                    out.y = encode4<FMT, F, true>(x[4], x[5], x[6], x[7], s, r);
+                    out.z = encode4<FMT, F, true>(y[0], y[1], y[2], y[3], s, r);
+                    out.w = encode4<FMT, F, true>(y[4], y[5], y[6], y[7], s, r);
+                };
+                if (__ballot(!ok) == 0) run(std::true_type{});
+                else run(std::false_type{});
+            }
+            if (used[i])
+                *reinterpret_cast<uint4*>(p.k_cache + page * p.kc_page + h[i] * p.kc_head +
+                                          ((d0[i] / E) * PAGE + pos) * 16) = out;
+        }
+    }
+
+    const float s = FMT != BF16 && p.v_scale ? p.v_scale[vh] : 1.0f;
+    const float r = FMT != BF16 ? __fdiv_rn(1.0f, s) : 1.0f;
+    const bool scale_ok = s >= kScaleMin && s <= kScaleMax;
+    // One token's two values to its slot.
+    const auto store_alone = [&](uint32_t x, int slot, bool fast) __attribute__((always_inline)) {
+        uint8_t* dst = v_dst + (slot / PAGE) * p.vc_page + (slot % PAGE) * ES;
+        if constexpr (FMT == BF16) {
+            *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(x);
+            *reinterpret_cast<uint16_t*>(dst + PAGE * ES) = static_cast<uint16_t>(x >> 16);
+        } else {
+            float a, b;
+            unpack_pair<IN>(x, a, b);
+            const uint32_t codes = fast ? encode4<FMT, true, true>(a, b, 0.0f, 0.0f, s, r)
+                                        : encode<FMT>(a, s, true) | encode<FMT>(b, s, true) << 8;
+            dst[0] = static_cast<uint8_t>(codes);
+            dst[PAGE] = static_cast<uint8_t>(codes >> 8);
+        }
+    };
+    if (w.run >= 0) {
+        const int slot = __builtin_amdgcn_readfirstlane(w.slot(w.run, first));
+        uint8_t* dst = v_dst + (slot / PAGE) * p.vc_page;
+        if constexpr (FMT == BF16) {
+            quiet_pairs(v);
+            uint32_t lo[8], hi[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                lo[j] = __builtin_amdgcn_perm(v[2 * j + 1], v[2 * j], 0x05040100u);
+                hi[j] = __builtin_amdgcn_perm(v[2 * j + 1], v[2 * j], 0x07060302u);
+            }
+            if (v_used) {
+                uint4* to = reinterpret_cast<uint4*>(dst);
+                to[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+                to[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
+                to[2] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                to[3] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
+            }
+        } else {
+            uint32_t m = 0;
+#pragma unroll
+            for (int j = 0; j < PAGE; ++j) m = max_pair(m, v[j] & 0x7FFF7FFFu);
+            const bool ok = scale_ok && magnitude_within<IN>(max(m & 0xFFFFu, m >> 16));
+            if (__ballot(!ok) == 0) {
+                uint32_t lo[4], hi[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float a[4], b[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) unpack_pair<IN>(v[4 * j + i], a[i], b[i]);
+                    lo[j] = encode4<FMT, true, true>(a[0], a[1], a[2], a[3], s, r);
+                    hi[j] = encode4<FMT, true, true>(b[0], b[1], b[2], b[3], s, r);
+                }
+                if (v_used) {
+                    uint4* to = reinterpret_cast<uint4*>(dst);
+                    to[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+                    to[1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                }
+            } else if (v_used) {
+                for (int j = 0; j < PAGE; ++j)
+                    store_alone(*reinterpret_cast<const uint32_t*>(v_src + (w.run + j) * p.sv_t), slot + j, false);
+            }
+        }
+    }
+    if (w.rest != 0) {
+        uint32_t m = 0;
+        if (w.run >= 0) load_rest();
+        if constexpr (FMT == BF16) quiet_pairs(v);
+#pragma unroll
+        for (int j = 0; j < PAGE; ++j) m = max_pair(m, v[j] & 0x7FFF7FFFu);
+        const bool ok = scale_ok && magnitude_within<IN>(max(m & 0xFFFFu, m >> 16));
+        if (FMT == BF16 || __ballot(!ok) == 0) {
+#pragma unroll
+            for (int j = 0; j < PAGE; ++j) {
+                const int slot = __builtin_amdgcn_readlane(w.slots, j + 15);
+                if ((w.rest >> j & 1) && v_used) store_alone(v[j], slot, true);
+            }
+        } else if (v_used) {
+            for (int j = 0; j < PAGE; ++j) {
+                const int slot = __builtin_amdgcn_readlane(w.slots, j + 15);
+                if (w.rest >> j & 1)
+                    store_alone(*reinterpret_cast<const uint32_t*>(v_src + (first + j) * p.sv_t), slot, false);
+            }
+        }
+    }
+}
+
+// Whether paged_append_window_kernel takes a call: 16-byte loads of the states, and a format it has an instance for.
+bool append_windows(const AppendParams& p) {
+    const bool formats = p.cache_format == BF16 ? p.in_format == BF16 : p.in_format == BF16 || p.in_format == FP16;
+    return formats && static_cast<int64_t>(p.kv_heads) * p.head_dim <= 65535 * 128 && ((p.sk_t | p.sk_h | p.sv_t | p.sv_h) & 7) == 0 &&
+           ((reinterpret_cast<uintptr_t>(p.k_new) | reinterpret_cast<uintptr_t>(p.v_new) |
+             reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 15) == 0;
 }
 
 // The append with Quest's metadata kept on the device, in one launch: workgroups below `tokens` append a token each;
@@ -332,6 +508,21 @@ __global__ void scales_from_absmax_kernel(const uint32_t* absmax_bits, int heads
 
 int paged_append(const AppendParams& p, hipStream_t stream) {
     if (p.tokens == 0) return 0;
+    if (append_windows(p)) {
+        dim3 grid, block;
+        window_launch(p.tokens, static_cast<int64_t>(p.kv_heads) * p.head_dim, grid, block);
+        const auto launch = [&](auto fmt, auto in) {
+            hipLaunchKernelGGL((paged_append_window_kernel<fmt.value, in.value>), grid, block, 0, stream, p);
+        };
+        const std::integral_constant<int, BF16> bf16;
+        const std::integral_constant<int, FP16> fp16;
+        const std::integral_constant<int, FP8_E4M3> e4m3;
+        const std::integral_constant<int, FP8_E5M2> e5m2;
+        if (p.cache_format == BF16) launch(bf16, bf16);
+        else if (p.cache_format == FP8_E4M3) p.in_format == BF16 ? launch(e4m3, bf16) : launch(e4m3, fp16);
+        else p.in_format == BF16 ? launch(e5m2, bf16) : launch(e5m2, fp16);
+        return check_launch("paged_append_window_kernel");
+    }
     dim3 grid(p.tokens);
     switch (p.cache_format) {
         case BF16: hipLaunchKernelGGL(paged_append_kernel<BF16>, grid, dim3(256), 0, stream, p); break;

@@ -201,7 +201,7 @@ def packed_mask(mask: torch.Tensor | None, batch: int, q_heads: int, queries: in
 
 def cached_workspace(nbytes: int, counters: int, device: torch.device) -> torch.Tensor:
     """The workspace of ``device``'s current stream used when the caller passes none (see :class:`CachedWorkspace`)."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, _lib.stream_of(device))
     return _workspaces.setdefault(key, CachedWorkspace()).take(nbytes, counters, device)
 
 

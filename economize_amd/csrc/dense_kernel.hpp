@@ -185,6 +185,14 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8& hi, bf16x8& 
     }
 }
 
+// ds_read_b64_tr_b16: the 16 lanes of a group name four rows of 16 elements, lane 4 k + q the eight bytes of row k's
+// elements 4 q .. 4 q + 3; lane i receives element i of the four rows.
+__device__ __forceinline__ uint2 transpose_read(const uint8_t* lds) {
+    typedef short i16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(
+        uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(lds)));
+}
+
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
@@ -253,14 +261,16 @@ __device__ inline float sink_weight(float m, float l, float sink, float& inv) {
 // Eight codes of channels c .. c + 7 packed along bytes (channel c + i at bit i BITS of x), as exact floats. The
 // codes are spread one per byte (even channels in lo, odd ones in hi); a code below 16 in a byte is the e4m3 pattern
 // of code 2^-9, which v_cvt_scalef32_pk_f32_fp8 with scale 2^9 turns into the exact float, two bytes at a time.
+// For 2-bit codes select names the half of x that holds them.
+constexpr uint32_t kLowHalf = 0x0C010C00u, kHighHalf = 0x0C030C02u;
 template <int BITS>
-__device__ __forceinline__ void cell_codes8(uint32_t x, float (&c)[8]) {
+__device__ __forceinline__ void cell_codes8(uint32_t x, float (&c)[8], uint32_t select = kLowHalf) {
     uint32_t lo, hi;
     if constexpr (BITS == 4) {  // nibbles: channel i at bit 4 i
         lo = x & 0x0F0F0F0Fu;          // channels 0, 2, 4, 6
         hi = (x >> 4) & 0x0F0F0F0Fu;   // channels 1, 3, 5, 7
-    } else {  // 2-bit fields of the low 16 bits: channel i at bit 2 i
-        const uint32_t u = __builtin_amdgcn_perm(0u, x, 0x0C010C00u);  // bytes: x.byte0, 0, x.byte1, 0
+    } else {  // 2-bit fields of a half: channel i at bit 2 i
+        const uint32_t u = __builtin_amdgcn_perm(0u, x, select);  // the half's bytes as byte 0 and byte 2
         const uint32_t v = (u | (u << 4)) & 0x0F0F0F0Fu;                // bytes: channels 0-1, 2-3, 4-5, 6-7
         lo = v & 0x03030303u;          // channels 0, 2, 4, 6
         hi = (v >> 2) & 0x03030303u;   // channels 1, 3, 5, 7
@@ -382,11 +392,12 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
     const int qi = r_ok ? qi0 : 0;
     const int h = kvh * p.groups + gq;
 
-    // the query operand: row r, channels 32 j + 8 g .. (zero past the head dim and for rows past the group)
+    // the query operand: row r, channels 32 j + 8 g .. (zero past the head dim and for rows past the group); codes:
+    // channels 32 g + 8 j .., so that a lane's key codes follow each other in the cell (one load, not one per j)
     bf16x8 qh[KS], ql[KS];
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
-        const int c = 32 * j + 8 * g;
+        const int c = CB != 0 ? 32 * g + 8 * j : 32 * j + 8 * g;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             qh[j][i] = static_cast<__bf16>(0.0f);
@@ -524,6 +535,7 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
     };
     // causal: the last q_count keys of the row are its queries' own tokens
     const int causal_limit = p.causal ? row_keys - q_count + qi + 1 : row_keys;
+    const int all_see = __builtin_amdgcn_readfirstlane(p.causal ? row_keys - q_count + 1 : row_keys);  // of every query
     auto mask_col = [&](int t) __attribute__((always_inline)) -> int64_t {
         if (p.qp_list) return quest_slot(t);
         return t < count ? min(max(gidx[t], 0), p.dense_keys - 1) : start + t - count;
@@ -546,10 +558,23 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
     struct Keys {
         uint4 k[CB != 0 ? 1 : 2][CB != 0 ? 1 : KS][KW];
         uint32_t m[MASKED ? 8 : 1];
-        uint32_t kc[2][CB != 0 ? KS : 1];  // codes: the code word of the lane's channels 32 j + 8 g .. of its key v
+        uint32_t kc[2][CB != 0 ? CB : 1];  // codes: the code words of the lane's channels 32 g .. 32 g + 31 of its key v
         uint32_t kf[2];                    // codes: the flag byte of its key v
         int64_t h0, h1;                    // codes: the tile's half offsets (the next tile's issue moves cell_h*)
     };
+    // codes: the lane's byte offsets from the tile's first cell: its value token's cell and its half of the value codes,
+    // its aux cell, its keys' cells and its words of their codes
+    int64_t cell_v = 0, cell_vcodes = 0, cell_aux = 0, cell_k[2] = {0, 0}, cell_kcodes[2] = {0, 0};
+    if constexpr (CB != 0) {
+        cell_v = (lane >> 1) * p.sc_token;
+        cell_vcodes = cell_v + 16 * (CB / 2) * (lane & 1);
+        cell_aux = (lane & 31) * p.sc_token;
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            cell_k[v] = (8 * (n >> 2) + 4 * v + (n & 3)) * p.sc_token;
+            cell_kcodes[v] = cell_k[v] + 4 * CB * g;
+        }
+    }
     // Every load is issued unconditionally at a clamped address (a key past the split reads the split's last key, a
     // channel past the dims reads channel 0) and what it must not contribute is zeroed where it is used: every path
     // through the loop then issues the same loads, and the wait before a tile's use leaves the younger tile's loads
@@ -560,23 +585,31 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
         if constexpr (CB != 0) {
             K.h0 = cell_h0;
             K.h1 = cell_h1;
-            const uint8_t* vc = cell_row(min(t0 + (lane >> 1), t_end - 1));
+            // The tile's 32 cells follow each other in one page (page_size is a multiple of 32): a wave-uniform base and
+            // the lane's offsets from it. Cells past the row's keys are read too (in the page), their keys hidden and
+            // their values zeroed below; a visible key's group aux may sit in one.
+            const uint8_t* tile = p.cells + cell_h0;
 #pragma unroll
             for (int i = 0; i < (CB == 4 ? 2 : 1); ++i)
-                vcw[i] = *reinterpret_cast<const uint4*>(vc + p.cell_off_vc + 16 * (CB / 2) * (lane & 1) + 16 * i);
-            vsz = *reinterpret_cast<const uint4*>(vc + p.cell_off_vs);
-            vfl = *(vc + p.cell_off_flag + 1);
-            // (every cell of the tile's key group: the tile's 32 cells lie in one page, page_size being a multiple
-            // of 32, and a visible key's group aux may sit in a cell past the row's keys)
-            vaux = *reinterpret_cast<const uint4*>(cell_row(t0 + (lane & 31)) + p.cell_off_ka);
+                vcw[i] = *reinterpret_cast<const uint4*>(tile + p.cell_off_vc + cell_vcodes + 16 * i);
+            vsz = *reinterpret_cast<const uint4*>(tile + p.cell_off_vs + cell_v);
+            vfl = *(tile + p.cell_off_flag + 1 + cell_v);
+            vaux = *reinterpret_cast<const uint4*>(tile + p.cell_off_ka + cell_aux);
 #pragma unroll
             for (int v = 0; v < 2; ++v) {
-                const uint8_t* krow = cell_row(min(t0 + 8 * (n >> 2) + 4 * v + (n & 3), t_end - 1));
-                K.kf[v] = *(krow + p.cell_off_flag);
-#pragma unroll
-                for (int j = 0; j < KS; ++j)
-                    K.kc[v][j] = *reinterpret_cast<const uint32_t*>(
-                        krow + p.cell_off_kc + (CB == 2 ? 4 * (2 * j + (g >> 1)) : 16 * j + 4 * g));
+                K.kf[v] = *(tile + p.cell_off_flag + cell_k[v]);
+                const uint8_t* codes = tile + p.cell_off_kc + cell_kcodes[v];
+                if constexpr (CB == 2) {
+                    const uint2 x = *reinterpret_cast<const uint2*>(codes);
+                    K.kc[v][0] = x.x;
+                    K.kc[v][CB - 1] = x.y;
+                } else {
+                    const uint4 x = *reinterpret_cast<const uint4*>(codes);
+                    K.kc[v][0] = x.x;
+                    K.kc[v][1] = x.y;
+                    K.kc[v][CB - 2] = x.z;
+                    K.kc[v][CB - 1] = x.w;
+                }
             }
             return;
         }
@@ -848,10 +881,9 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
                 // (selects, not an index by the lane's half: a vector indexed at run time goes to scratch)
                 const float sc = static_cast<float>(hh ? sz[2 + q / 4] : sz[q / 4]);
                 const float zr = static_cast<float>(hh ? sz[6 + q / 4] : sz[4 + q / 4]);
-                const uint32_t x = CB == 2 ? (word_of(vcw[0], q >> 1) >> (16 * (q & 1))) & 0xFFFFu
-                                           : word_of(vcw[CB == 4 ? (q >> 2) : 0], q & 3);
+                const uint32_t x = CB == 2 ? word_of(vcw[0], q >> 1) : word_of(vcw[CB == 4 ? (q >> 2) : 0], q & 3);
                 float c[8], scs[8], zrs[8];
-                cell_codes8<CB>(x, c);
+                cell_codes8<CB>(x, c, q & 1 ? kHighHalf : kLowHalf);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     scs[i] = sc;
@@ -870,6 +902,9 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
                     *reinterpret_cast<uint4*>(dst + 16 * q) = vok ? out[q] : make_uint4(0, 0, 0, 0);
+            } else if (t0 + TK <= t_end) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) *reinterpret_cast<uint4*>(dst + 16 * q) = out[q];
             } else {
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
@@ -900,8 +935,8 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
         // ---- S^T = K Q^T (key channels past the head dim zeroed) ----
         f32x4 s[2];
         if constexpr (CB != 0) {
-            // the lane's key scales and zero points (channels 32 j + 8 g ..: entries of the group's aux in the slots
-            // of cells 4 j + g and 16 + 4 j + g), then the keys from their codes, or their dense entries where the
+            // the lane's key scales and zero points (channels 32 g + 8 j ..: entries of the group's aux in the slots
+            // of cells 4 g + j and 16 + 4 g + j), then the keys from their codes, or their dense entries where the
             // flag is not 1 (a rare branch that keeps its loads and their uses to itself)
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the aux stores of this tile (one wave: in order)
             auto scores = [&](bool dense) __attribute__((always_inline)) {
@@ -909,13 +944,12 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
                 for (int v = 0; v < 2; ++v) s[v] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < KS; ++j) {
-                    const f16x8 sj = *reinterpret_cast<const f16x8*>(auxl + 16 * (4 * j + g));
-                    const f16x8 zj = *reinterpret_cast<const f16x8*>(auxl + 16 * (16 + 4 * j + g));
+                    const f16x8 sj = *reinterpret_cast<const f16x8*>(auxl + 16 * (4 * g + j));
+                    const f16x8 zj = *reinterpret_cast<const f16x8*>(auxl + 16 * (16 + 4 * g + j));
 #pragma unroll
                     for (int v = 0; v < 2; ++v) {
-                        const uint32_t x = CB == 2 ? (K.kc[v][j] >> (16 * (g & 1))) & 0xFFFFu : K.kc[v][j];
                         float c[8];
-                        cell_codes8<CB>(x, c);
+                        cell_codes8<CB>(K.kc[v][CB == 2 ? j / 2 : j], c, j & 1 ? kHighHalf : kLowHalf);
                         bf16x8 kh;  // (the fp16 scales widened inside each product: v_fma_mix_f32)
 #pragma unroll
                         for (int i = 0; i < 8; ++i)
@@ -925,7 +959,7 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
                             const int tk = min(t0 + 8 * (n >> 2) + 4 * v + (n & 3), t_end - 1);
                             const uint8_t* row = p.cells + ((tk >> 4) & 1 ? K.h1 : K.h0) +
                                                  static_cast<int64_t>(tk & 15) * p.sc_token;
-                            kh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + 2 * (32 * j + 8 * g)));
+                            kh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + 2 * (32 * g + 8 * j)));
                         }
                         s[v] = mfma(kh, qh[j], s[v]);
                     }
@@ -966,14 +1000,6 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
         }
         }
         // ---- scores in log2 units, masked: lane (n, g) holds keys t0 + 8 g + 4 v + i of row r ----
-        uint32_t vis = 0;  // bit 4 v + i
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int t = t0 + 8 * g + e;
-            bool ok = r_ok && t < t_end && t < causal_limit;
-            if constexpr (MASKED) ok = ok && (K.m[e] & 0xFFu) != 0;
-            vis |= ok ? 1u << e : 0u;
-        }
         float tile_max = -INFINITY;
         // the soft cap tested once per tile, not per score (the compiler keeps a uniform test inside an unrolled loop)
         if (p.softcap > 0.0f) {
@@ -987,16 +1013,24 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
 #pragma unroll
                 for (int i = 0; i < 4; ++i) s[v][i] *= score_scale;
         }
+        // (a tile every query sees needs no masking; a lane without a query row keeps weights nobody stores)
+        if (MASKED || t0 + TK > all_see) {
+#pragma unroll
+            for (int v = 0; v < 2; ++v)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = t0 + 8 * g + 4 * v + i;
+                    bool ok = r_ok && t < t_end && t < causal_limit;
+                    if constexpr (MASKED) ok = ok && (K.m[4 * v + i] & 0xFFu) != 0;
+                    s[v][i] = ok ? s[v][i] : -INFINITY;
+                }
+        }
 #pragma unroll
         for (int v = 0; v < 2; ++v)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float x = (vis >> (4 * v + i)) & 1u ? s[v][i] : -INFINITY;
-                s[v][i] = x;
-                tile_max = max_nan(tile_max, x);
-            }
+            tile_max = max_nan(max_nan(tile_max, max_nan(s[v][0], s[v][1])), max_nan(s[v][2], s[v][3]));
         // ---- online softmax, lazy rescaling (the reference maximum moves when a score exceeds it by 2^8) ----
-        if (__ballot(tile_max > m_i + 8.0f || m_i == -INFINITY) != 0) {
+        // (lanes without a query row do not ask for it: under a mask theirs would stay -inf and rescale every tile)
+        if (__ballot(r_ok && (tile_max > m_i + 8.0f || m_i == -INFINITY)) != 0) {
             const bool fresh = m_i == -INFINITY;
             const float m_new = fmaxf(m_i, group_max(tile_max));
             const float alpha = fresh ? 0.0f : __builtin_amdgcn_exp2f(m_i - m_new);
@@ -1028,6 +1062,13 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
             split8(pw, ph, pl);
         }
         // ---- O^T += V^T P^T: lane (n, g) supplies channel 16 nd + n of keys 8 g .. 8 g + 7 ----
+        // 16-bit values: two transposing LDS reads (ds_read_b64_tr_b16), each four rows of 16 channels held by a group of
+        // 16 lanes, in place of eight 2-byte reads and their packing: MEASURED
+        auto value_column = [&](int nd) __attribute__((always_inline)) {
+            const uint8_t* from = vtile + (8 * g + (n >> 2)) * ROW + 32 * nd + 8 * (n & 3);
+            const uint2 lo = transpose_read(from), hi = transpose_read(from + 4 * ROW);
+            return make_uint4(lo.x, lo.y, hi.x, hi.y);
+        };
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the tile's LDS stores (one wave: in order)
 #pragma unroll
         for (int nd = 0; nd < ND; ++nd) {
@@ -1035,12 +1076,11 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
             if (v0 + 16 * nd >= p.value_dim) break;
             if constexpr (H16) {
                 f16x8 vh16;
+                if constexpr (FMT == FP16) {
+                    vh16 = __builtin_bit_cast(f16x8, value_column(nd));
+                } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    if constexpr (FMT == FP16)
-                        vh16[e] = __builtin_bit_cast(_Float16,
-                                                     *reinterpret_cast<const uint16_t*>(vtile + (8 * g + e) * ROW + c * 2));
-                    else
+                    for (int e = 0; e < 8; ++e)
                         vh16[e] = static_cast<_Float16>(elem_f32<FMT>(vtile + (8 * g + e) * ROW + c * ES));
                 }
                 acc[nd] = mfma_h(vh16, ph16, acc[nd]);
@@ -1049,13 +1089,17 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
             }
             bf16x8 vh, vl;
             if constexpr (FMT == BF16) {  // the staged bits are the operand (no widening and rounding back)
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    vh[e] = __builtin_bit_cast(__bf16, *reinterpret_cast<const uint16_t*>(vtile + (8 * g + e) * ROW + c * 2));
+                vh = __builtin_bit_cast(bf16x8, value_column(nd));
             } else {
                 float x[8];
+                if constexpr (ES == 2) {
+                    const f16x8 column = __builtin_bit_cast(f16x8, value_column(nd));
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = elem_f32<FMT>(vtile + (8 * g + e) * ROW + c * ES);
+                    for (int e = 0; e < 8; ++e) x[e] = static_cast<float>(column[e]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] = elem_f32<FMT>(vtile + (8 * g + e) * ROW + c * ES);
+                }
                 split8(x, vh, vl);
             }
             acc[nd] = mfma(vh, ph, acc[nd]);

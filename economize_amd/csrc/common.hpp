@@ -100,7 +100,8 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // The larger of two pairs of 16-bit magnitudes.
 __device__ __forceinline__ uint32_t max_pair(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+    return __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
 }
 
 // The largest magnitude's bits in the four words' eight values, in the low half.

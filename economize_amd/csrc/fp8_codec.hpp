@@ -1,4 +1,5 @@
-// Bit-level float conversions shared by the kernels and the host: bf16 rounding and the fp8 encoder; division by a shared divisor.
+// Bit-level float conversions shared by the kernels and the host: bf16 rounding and the fp8 encoder;
+// division by a shared divisor.
 // Written without HIP headers so that the same code compiles for the CPU (its CPU test compiles it with g++).
 #pragma once
 

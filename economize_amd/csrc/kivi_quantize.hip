@@ -77,8 +77,8 @@ __global__ __launch_bounds__(256) void kivi_ring_kernel(KiviRingParams p) {
 // its row's ring and its place in it) and units of 128 channels over the KV heads, one wave each. Bound by moving the
 // states; the workgroup-per-token kernel is bound by its value stores, 2 bytes each at the ring's stride. Keys are copied
 // 16 bytes at a time; for values a lane holds two channels of a run's 16 tokens and stores 32 bytes of each; the four
-// waves of a workgroup take successive windows, so that they fill a value line together. 8 rows' 384 tokens x 8 KV heads, D = 128
-// (25 MB): 33 us by token, 8 us by windows.
+// waves of a workgroup take successive windows, so that they fill a value line together. 8 rows' 384 tokens x 8 KV
+// heads, D = 128 (25 MB): 33 us by token, 8 us by windows.
 __global__ __launch_bounds__(256) void kivi_ring_window_kernel(KiviRingParams p) {
     const int lane = threadIdx.x & 63;
     const int first = first_of_window();

@@ -38,9 +38,9 @@ __device__ inline uint8_t encode(float x, float scale, bool scaled) {
 // ---- encoding four values at a time -------------------------------------------------------------------------------
 //
 // What encode() computes, for bf16 and fp16 inputs: x / s as corrected_quotient and the hardware's round-to-nearest-even
-// conversion of two values per instruction, about 6 operations per value instead of 30. The quotient is IEEE division's for every 8- or 11-bit
-// significand of x and every fp32 significand of s (checked exhaustively) while nothing under- or overflows, which
-// kScaleMin <= s <= kScaleMax and |x| < 2^60 ensure down to |x| = 2^-64; a smaller |x| gives a quotient below 2^-23, a zero
+// conversion of two values per instruction, about 6 operations per value instead of 30. The quotient is IEEE
+// division's for every 8- or 11-bit significand of x and every fp32 significand of s (checked exhaustively) while
+// nothing under- or overflows, which kScaleMin <= s <= kScaleMax and |x| < 2^60 ensure down to |x| = 2^-64; a smaller |x| gives a quotient below 2^-23, a zero
 // of x's sign in both formats either way. The conversion equals f32_to_fp8 on every fp32 value up to the format's maximum
 // (checked on all of them). Values outside these limits (and NaN) take encode().
 constexpr float kScaleMin = 0x1p-40f, kScaleMax = 0x1p60f;
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(256) void paged_append_window_kernel(AppendParams p
 // Whether paged_append_window_kernel takes a call: 16-byte loads of the states, and a format it has an instance for.
 bool append_windows(const AppendParams& p) {
     const bool formats = p.cache_format == BF16 ? p.in_format == BF16 : p.in_format == BF16 || p.in_format == FP16;
-    return formats && static_cast<int64_t>(p.kv_heads) * p.head_dim <= 65535 * 128 && ((p.sk_t | p.sk_h | p.sv_t | p.sv_h) & 7) == 0 &&
+    return formats && static_cast<int64_t>(p.kv_heads) * p.head_dim <= 65535 * 128 &&
+           ((p.sk_t | p.sk_h | p.sv_t | p.sv_h) & 7) == 0 &&
            ((reinterpret_cast<uintptr_t>(p.k_new) | reinterpret_cast<uintptr_t>(p.v_new) |
              reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 15) == 0;
 }

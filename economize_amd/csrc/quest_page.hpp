@@ -24,8 +24,9 @@ __device__ inline float quest_decode_elem(const uint8_t* p, int i) {
     }
 }
 
-// The bounds of Quest page qp of (row b, KV head kvh) by one wave, any head dim, alignment and values: lane l holds token l % 16 of the runs l / 16,
-// l / 16 + 4, ... of every cache page of the Quest page; the 16 lanes of a run then reduce over the tokens.
+// The bounds of Quest page qp of (row b, KV head kvh) by one wave, any head dim, alignment and values: lane l holds
+// token l % 16 of the runs l / 16, l / 16 + 4, ... of every cache page of the Quest page; the 16 lanes of a run then
+// reduce over the tokens.
 template <int FMT>
 __device__ inline void quest_bounds_of_page(const BoundsParams& p, int b, int qp, int kvh, int lane) {
     constexpr int ES = FMT == BF16 ? 2 : 1;

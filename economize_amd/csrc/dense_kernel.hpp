@@ -323,6 +323,53 @@ __device__ __forceinline__ bf16x8 dequant_cell8(const float (&c)[8], const float
     return r;
 }
 
+// v_permlane32_swap / v_permlane16_swap: the upper two of a's four lane rows with the lower two of b's; a's odd lane rows
+// with b's even ones.
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+__device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// group_max without LDS (x swapped with itself leaves one side of a pair in either register).
+__device__ __forceinline__ float row_max(float x) {
+    uint32_t a = f32_bits(x), b = a;
+    swap_rows(a, b);
+    x = max_nan(bits_f32(a), bits_f32(b));
+    a = b = f32_bits(x);
+    swap_halves(a, b);
+    return max_nan(bits_f32(a), bits_f32(b));
+}
+
+// The key codes of a 128-channel cell as lane (n, g) needs them, channels 32 j + 8 g .., from the words it loaded,
+// channels 32 g .. 32 g + 31 (one load per key): the 8-channel runs transposed over the four lane rows. 4 bits: run j is
+// out[j]. 2 bits (a run is a half word): run j is half j / 2 of out[j % 2].
+template <int BITS>
+__device__ __forceinline__ void key_code_words(const uint32_t (&in)[BITS], uint32_t (&out)[BITS]) {
+    uint32_t w[BITS];
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) w[i] = in[i];
+    if constexpr (BITS == 4) {
+        swap_halves(w[0], w[2]);
+        swap_halves(w[1], w[3]);
+        swap_rows(w[0], w[1]);
+        swap_rows(w[2], w[3]);
+#pragma unroll
+        for (int i = 0; i < BITS; ++i) out[i] = w[i];
+    } else {
+        swap_halves(w[0], w[1]);
+        out[0] = __builtin_amdgcn_perm(w[1], w[0], 0x05040100u);
+        out[1] = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
+        swap_rows(out[0], out[1]);
+    }
+}
+
 __device__ __forceinline__ uint32_t word_of(uint4 x, int i) {
     return i == 0 ? x.x : (i == 1 ? x.y : (i == 2 ? x.z : x.w));
 }
@@ -392,12 +439,11 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
     const int qi = r_ok ? qi0 : 0;
     const int h = kvh * p.groups + gq;
 
-    // the query operand: row r, channels 32 j + 8 g .. (zero past the head dim and for rows past the group); codes:
-    // channels 32 g + 8 j .., so that a lane's key codes follow each other in the cell (one load, not one per j)
+    // the query operand: row r, channels 32 j + 8 g .. (zero past the head dim and for rows past the group)
     bf16x8 qh[KS], ql[KS];
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
-        const int c = CB != 0 ? 32 * g + 8 * j : 32 * j + 8 * g;
+        const int c = 32 * j + 8 * g;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             qh[j][i] = static_cast<__bf16>(0.0f);
@@ -541,6 +587,11 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
         return t < count ? min(max(gidx[t], 0), p.dense_keys - 1) : start + t - count;
     };
 
+    // How far a score may pass the reference maximum before it moves: 2^8 in a block of 16 query rows, where some row
+    // finds a larger score in most tiles. A block with fewer rows (a decode step) takes the maximum itself, so that its
+    // largest weight, 1, is exact in the bf16 (fp16) operand of the value product (2-bit cells, 16 rows x 8192 tokens of
+    // 4 query rows: 70.2 us, 69.2 with 2^8 here too).
+    const float slack = __ballot(!r_ok) != 0 ? 0.0f : 8.0f;
     float m_i = -INFINITY, l_i = 0.0f;
     f32x4 acc[ND];
 #pragma unroll
@@ -586,9 +637,10 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
             K.h0 = cell_h0;
             K.h1 = cell_h1;
             // The tile's 32 cells follow each other in one page (page_size is a multiple of 32): a wave-uniform base and
-            // the lane's offsets from it (with the masks of full tiles left out, 80.3 -> 76.9 us; with a lane's key codes
-            // in one load, 68.1). Cells past the row's keys are read too (in the page), their keys hidden and
-            // their values zeroed below; a visible key's group aux may sit in one.
+            // the lane's offsets from it (with the masks of full tiles left out, 80.3 -> 76.9 us at 16 rows x 8192 tokens,
+            // 2 bits; with a lane's key codes in one load and their runs exchanged between lanes, 70.2). Cells past the
+            // row's keys are read too (in the page), their keys hidden and their values zeroed below; a visible key's
+            // group aux may sit in one.
             const uint8_t* tile = p.cells + cell_h0;
 #pragma unroll
             for (int i = 0; i < (CB == 4 ? 2 : 1); ++i)
@@ -936,21 +988,24 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
         // ---- S^T = K Q^T (key channels past the head dim zeroed) ----
         f32x4 s[2];
         if constexpr (CB != 0) {
-            // the lane's key scales and zero points (channels 32 g + 8 j ..: entries of the group's aux in the slots
-            // of cells 4 g + j and 16 + 4 g + j), then the keys from their codes, or their dense entries where the
+            // the lane's key scales and zero points (channels 32 j + 8 g ..: entries of the group's aux in the slots
+            // of cells 4 j + g and 16 + 4 j + g), then the keys from their codes, or their dense entries where the
             // flag is not 1 (a rare branch that keeps its loads and their uses to itself)
+            uint32_t kc[2][CB];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) key_code_words<CB>(K.kc[v], kc[v]);
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the aux stores of this tile (one wave: in order)
             auto scores = [&](bool dense) __attribute__((always_inline)) {
 #pragma unroll
                 for (int v = 0; v < 2; ++v) s[v] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < KS; ++j) {
-                    const f16x8 sj = *reinterpret_cast<const f16x8*>(auxl + 16 * (4 * g + j));
-                    const f16x8 zj = *reinterpret_cast<const f16x8*>(auxl + 16 * (16 + 4 * g + j));
+                    const f16x8 sj = *reinterpret_cast<const f16x8*>(auxl + 16 * (4 * j + g));
+                    const f16x8 zj = *reinterpret_cast<const f16x8*>(auxl + 16 * (16 + 4 * j + g));
 #pragma unroll
                     for (int v = 0; v < 2; ++v) {
                         float c[8];
-                        cell_codes8<CB>(K.kc[v][CB == 2 ? j / 2 : j], c, j & 1 ? kHighHalf : kLowHalf);
+                        cell_codes8<CB>(kc[v][CB == 2 ? j & 1 : j], c, j / 2 ? kHighHalf : kLowHalf);
                         bf16x8 kh;  // (the fp16 scales widened inside each product: v_fma_mix_f32)
 #pragma unroll
                         for (int i = 0; i < 8; ++i)
@@ -960,7 +1015,7 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
                             const int tk = min(t0 + 8 * (n >> 2) + 4 * v + (n & 3), t_end - 1);
                             const uint8_t* row = p.cells + ((tk >> 4) & 1 ? K.h1 : K.h0) +
                                                  static_cast<int64_t>(tk & 15) * p.sc_token;
-                            kh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + 2 * (32 * g + 8 * j)));
+                            kh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(row + 2 * (32 * j + 8 * g)));
                         }
                         s[v] = mfma(kh, qh[j], s[v]);
                     }
@@ -1029,11 +1084,11 @@ __global__ __launch_bounds__(64, DP > 256 ? 1 : 2) void dense_split_kernel(Dense
 #pragma unroll
         for (int v = 0; v < 2; ++v)
             tile_max = max_nan(max_nan(tile_max, max_nan(s[v][0], s[v][1])), max_nan(s[v][2], s[v][3]));
-        // ---- online softmax, lazy rescaling (the reference maximum moves when a score exceeds it by 2^8) ----
+        // ---- online softmax, lazy rescaling (the reference maximum moves when a score exceeds it by 2^slack) ----
         // (lanes without a query row do not ask for it: under a mask theirs would stay -inf and rescale every tile)
-        if (__ballot(r_ok && (tile_max > m_i + 8.0f || m_i == -INFINITY)) != 0) {
+        if (__ballot(r_ok && (tile_max > m_i + slack || m_i == -INFINITY)) != 0) {
             const bool fresh = m_i == -INFINITY;
-            const float m_new = fmaxf(m_i, group_max(tile_max));
+            const float m_new = fmaxf(m_i, row_max(tile_max));
             const float alpha = fresh ? 0.0f : __builtin_amdgcn_exp2f(m_i - m_new);
             l_i *= alpha;
 #pragma unroll

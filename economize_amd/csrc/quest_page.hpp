@@ -206,17 +206,25 @@ __device__ __forceinline__ void quest_bounds_pages(const BoundsParams& p, int b,
         fold_min<0xB1, F>(v2, b0, v1);       // quad_perm 1 0 3 2
         const int qp = q0 + i / p.span;
         bool nan = false;
-        uint16_t* out = (kind ? p.kmax : p.kmin) + b * p.sb_b + kvh * p.sb_h + qp * p.sb_p;
-        const int first = (b2 * 4 + b1 * 2 + b0) * F;
+        i16x2 x[F];  // ordered bf16 pairs
 #pragma unroll
         for (int j = 0; j < F; ++j) {
-            const i16x2 x = as_i16x2(kind ? ~as_u32(v1[j]) : as_u32(v1[j]));  // ordered bf16 pairs
-            nan |= kind ? x[0] > 0x7F80 || x[1] > 0x7F80 : x[0] < -0x7F81 || x[1] < -0x7F81;
-            const int v = first + j;
-            const int channel = (4 * (v / DPL) + g) * (2 * DPL) + 2 * (v % DPL);
-            if (held) *reinterpret_cast<uint32_t*>(out + channel) = as_u32(ordered_bf16(x));
+            x[j] = as_i16x2(kind ? ~as_u32(v1[j]) : as_u32(v1[j]));
+            nan |= kind ? x[j][0] > 0x7F80 || x[j][1] > 0x7F80 : x[j][0] < -0x7F81 || x[j][1] < -0x7F81;
         }
-        if (held && __ballot(nan) != 0) quest_bounds_of_page<FMT>(p, b, qp, kvh, lane);
+        // (one of the two writes the page: the other's lanes would store to the same bounds in no stated order)
+        if (held && __ballot(nan) != 0) {
+            quest_bounds_of_page<FMT>(p, b, qp, kvh, lane);
+        } else if (held) {
+            uint16_t* out = (kind ? p.kmax : p.kmin) + b * p.sb_b + kvh * p.sb_h + qp * p.sb_p;
+            const int first = (b2 * 4 + b1 * 2 + b0) * F;
+#pragma unroll
+            for (int j = 0; j < F; ++j) {
+                const int v = first + j;
+                const int channel = (4 * (v / DPL) + g) * (2 * DPL) + 2 * (v % DPL);
+                *reinterpret_cast<uint32_t*>(out + channel) = as_u32(ordered_bf16(x[j]));
+            }
+        }
         held = true;
     }
 }

@@ -1,7 +1,7 @@
 """Quest page bounds over a prompt's pages (``paged_page_bounds``, ``QuestState.refresh``) where the packed reduction
 can go wrong: every head dim it has an instance for and ones it has not, pages of several cache pages, more cache pages
-than one window of the block table, rows of different lengths, signed zeros, infinities and NaN (which the minimum and
-maximum skip), missing pages (left untouched) and bounds at an odd element offset. Exact: whole values."""
+than one window of the block table, rows of different lengths, signed zeros (-0 below +0), infinities and NaN (which the
+minimum and maximum skip), missing pages (left untouched) and bounds at an odd element offset. Exact: the bounds' bits."""
 
 from __future__ import annotations
 
@@ -25,6 +25,11 @@ def _cache(dtype, dim: int, pages: int, seed: int):
     at = torch.rand(keys.shape, generator=gen)
     for k, special in enumerate((0.0, -0.0, 448.0, -448.0, 1e-3, -1e-3)):
         keys = torch.where((at > 0.01 * k) & (at < 0.01 * (k + 1)), torch.tensor(special), keys)
+    # every fourth page has a zero of some sign for its minimum in most channels, the next one for its maximum
+    zeros = torch.where(torch.rand(keys.shape, generator=gen) < 0.5, 0.0, -0.0)
+    halves = torch.where(torch.rand(keys.shape, generator=gen) < 0.3, zeros, keys.abs())
+    kind = (torch.arange(total) % 4).view(-1, 1, 1, 1, 1)
+    keys = torch.where(kind == 1, halves, torch.where(kind == 2, -halves, keys))
     # pages 0 .. total / 2 carry NaN of both signs, the others none
     nan = (at > 0.995) & (torch.arange(total) < total // 2).view(-1, 1, 1, 1, 1)
     stored = keys.to(dtype)
@@ -44,14 +49,22 @@ def _cache(dtype, dim: int, pages: int, seed: int):
     return cache, table.cuda(), dense.numpy()
 
 
+def _ordered(bits: np.ndarray) -> np.ndarray:
+    return bits ^ ((bits >> 15) & np.int16(0x7FFF))
+
+
 def _expected(dense: np.ndarray, table: np.ndarray, quest_page: int, q0: int, q1: int):
-    """fp32 bounds of Quest pages [q0, q1) as the kernel's fminf / fmaxf take them, and which pages are held."""
+    """bf16 bits of the bounds of Quest pages [q0, q1), the infinities of no key where all are NaN, and which pages are
+    held. The minimum and maximum are those of the bits as int16 in the order of the floats (the map is its inverse)."""
     span = quest_page // 16
     x = dense[:, :, q0 * quest_page: q1 * quest_page].reshape(B, HKV, q1 - q0, quest_page, -1)
     held = (table[:, q0 * span: q1 * span].reshape(B, q1 - q0, span) >= 0).all(axis=2)
-    lo = np.where(np.isnan(x), np.inf, x).min(axis=3)
-    hi = np.where(np.isnan(x), -np.inf, x).max(axis=3)
-    return lo, hi, held[:, None, :, None]
+    bits = (x.view(np.uint32) >> 16).astype(np.uint16).view(np.int16)  # the keys are bf16 values
+    ordered = _ordered(bits)
+    top = np.int16(0x7F80)  # infinity; its negative's place is ~top
+    lo = np.where(np.isnan(x), top, ordered).min(axis=3)
+    hi = np.where(np.isnan(x), ~top, ordered).max(axis=3)
+    return _ordered(lo), _ordered(hi), held[:, None, :, None]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn, torch.float8_e5m2])
@@ -69,8 +82,8 @@ def test_bounds_of_a_prompt(dtype, dim, quest_page, quest_pages) -> None:
         lo, hi, held = want
         for b, n in enumerate(limit):
             for got, ref in ((kmin, lo), (kmax, hi)):
-                ref = np.where(held[b], ref[b], 0.0)[:, :n]
-                np.testing.assert_array_equal(got[b, :, :n].float().cpu().numpy(), ref)
+                ref = np.where(held[b], ref[b], np.int16(0))[:, :n]
+                np.testing.assert_array_equal(got[b, :, :n].view(torch.int16).cpu().numpy(), ref)
 
     check(*paged_page_bounds(cache, table, 0, quest_pages, quest_page))
     # into bounds that start at an odd element: 2-byte stores only

@@ -7,9 +7,10 @@
 // modules/kv_cache.py:13-27). The per-head scale is the reference's static_scales rule (fp8.py:130-133) over each
 // KV head's absolute maximum.
 //
-// Layout of the caches: see paged_attention.hip. One workgroup per new token; a thread encodes 8 consecutive
-// channels of one head, so the key write is one 8-byte (fp8) or 16-byte (bf16) store into the token's 16-byte run,
-// and the value write scatters the 8 channels into their channel rows.
+// Layout of the caches: see paged_attention.hip. 16-bit states with aligned channels are appended by windows of 16 tokens
+// (paged_append_window_kernel); any others, and an append that keeps Quest's metadata, by one workgroup per new token: a
+// thread encodes 8 consecutive channels of one head, so the key write is one 8-byte (fp8) or 16-byte (bf16) store into
+// the token's 16-byte run, and the value write scatters the 8 channels into their channel rows.
 
 #include "common.hpp"
 #include "kv_quant.hpp"
@@ -39,10 +40,11 @@ __device__ inline uint8_t encode(float x, float scale, bool scaled) {
 //
 // What encode() computes, for bf16 and fp16 inputs: x / s as corrected_quotient and the hardware's round-to-nearest-even
 // conversion of two values per instruction, about 6 operations per value instead of 30. The quotient is IEEE
-// division's for every 8- or 11-bit significand of x and every fp32 significand of s (checked exhaustively) while
-// nothing under- or overflows, which kScaleMin <= s <= kScaleMax and |x| < 2^60 ensure down to |x| = 2^-64; a smaller |x| gives a quotient below 2^-23, a zero
-// of x's sign in both formats either way. The conversion equals f32_to_fp8 on every fp32 value up to the format's maximum
-// (checked on all of them). Values outside these limits (and NaN) take encode().
+// division's for every 8- or 11-bit significand of x and every fp32 significand of s (its CPU test compares them all)
+// while nothing under- or overflows, which kScaleMin <= s <= kScaleMax and |x| < 2^60 ensure down to |x| = 2^-64; a
+// smaller |x| gives a quotient below 2^-23, a zero of x's sign in both formats either way. The conversion rounds as
+// f32_to_fp8 does up to the format's maximum (the GPU test compares the two kernels on every 16-bit input, the ties of
+// both formats and their neighbours among them, at twelve scales). Values outside these limits (and NaN) take encode().
 constexpr float kScaleMin = 0x1p-40f, kScaleMax = 0x1p60f;
 
 template <int FMT>

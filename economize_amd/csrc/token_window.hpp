@@ -43,7 +43,14 @@ __device__ __forceinline__ TokenWindow token_window(int first, int tokens, int l
 // alone cost a wave up to 64 store requests each, so a call that does not fill the chip takes one wave per workgroup, and
 // so more compute units (128 tokens of different pages, 8 KV heads of 128 channels, fp8 pages / rings: 8.6 / 10.2 us by four
 // waves per workgroup, 6.0 / 6.2 by one, 4.7 / 5.4 with keys and values apart; 6.4 / 5.5 by the kernels of one workgroup
-// per token); longer ones take four, whose windows are successive.
+// per token); longer ones take four, whose windows are successive. By tokens (8 heads of 128, fp8 pages, us): one wave and
+// two passes, four waves, the kernel of one workgroup per token, for tokens alone in their pages, prompts of 30, prompts
+// of whole pages:
+//     512   alone   6.5  10.3   9.3    30   5.4   7.0   8.8    pages   4.1   5.1   8.8
+//    2048   alone  13.7  14.6  22.0    30   8.8   7.9  20.1    pages   5.0   5.7  19.7
+//    8192   alone  44.5  45.3  62.5    30  22.2  19.5  60.4    pages  12.6  12.1  60.6
+//   32768   alone   413   439   440    30  70.8  67.0   207    pages  41.2  40.5   206
+// and rings in runs of 64 at 32768: 99.5, 63.9, 417. The two forms cross between 2048 and 8192 tokens (1024 and 4096 waves).
 __device__ __forceinline__ int first_of_window() {
     return (blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 16;
 }

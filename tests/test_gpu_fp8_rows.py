@@ -1,6 +1,7 @@
 """The fp8 encode of bf16 and fp16 rows by 16-byte loads against the same values encoded as fp32 (the kernel that takes
 any row), bit for bit: head dims that leave lanes idle, token counts around a workgroup's rows, every scale mode, every
-16-bit pattern, scales outside the corrected quotient's limits, misaligned sources and destinations."""
+16-bit pattern, scales outside the corrected quotient's limits, misaligned sources, and destinations whose row stride the
+kernel takes (a multiple of 8 bytes) or leaves to the other one."""
 
 from __future__ import annotations
 
@@ -42,10 +43,12 @@ def test_rows(dtype, source, dim, tokens) -> None:
     _compare(x.transpose(1, 2).contiguous().transpose(1, 2), dtype, torch.tensor([0.5, 7e-4, 1.7], device="cuda"))
     odd = torch.empty(x.numel() + 1, dtype=source, device="cuda")[1:].view(x.shape).copy_(x)
     _compare(odd, dtype, torch.tensor([0.5, 7e-4, 1.7], device="cuda"))
-    buffer = torch.zeros(2, 3, tokens + 3, dim + 4, dtype=torch.uint8, device="cuda")
-    _encode(x, dtype, out=buffer[:, :, 2: 2 + tokens, :dim].view(dtype))
-    assert torch.equal(buffer[:, :, 2: 2 + tokens, :dim], _encode(x.float(), dtype))
-    assert not buffer[:, :, :2].any() and not buffer[:, :, 2 + tokens:].any() and not buffer[..., dim:].any()
+    for extra in (4, 8):
+        buffer = torch.full((2, 3, tokens + 3, dim + extra), 0x5A, dtype=torch.uint8, device="cuda")
+        _encode(x, dtype, out=buffer[:, :, 2: 2 + tokens, :dim].view(dtype))
+        want = torch.full_like(buffer, 0x5A)
+        want[:, :, 2: 2 + tokens, :dim] = _encode(x.float(), dtype)
+        assert torch.equal(buffer, want)
 
 
 @pytest.mark.parametrize("dtype", FORMATS)

@@ -123,7 +123,7 @@ __device__ inline bool quest_bounds_packed(const BoundsParams& p) {
 // wave writes the page's bounds with contiguous stores. The next cache page's loads are in flight while a page is
 // reduced, and the block table comes 64 entries per load. A page with a NaN (an extreme beyond infinity) is redone by
 // quest_bounds_of_page, whose fp32 minimum and maximum ignore NaN. 32,768 tokens of 64 (row, KV head) pairs, bf16, D =
-// 128 (604 MB): 120 us (5.0 TB/s), against 2123 us with a page reduced by 256 lane shuffles after dependent loads, in
+// 128 (604 MB): 121 us (5.0 TB/s), against 2123 us with a page reduced by 256 lane shuffles after dependent loads, in
 // eight waves per (row, KV head).
 template <int FMT, int D>
 __device__ __forceinline__ void quest_bounds_pages(const BoundsParams& p, int b, int kvh, int q0, int q1, int lane) {
